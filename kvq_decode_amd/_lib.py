@@ -6,26 +6,35 @@ check in the library runs before any HIP call. There is deliberately no fallback
 library is missing the import of the op fails loudly.
 """
 import ctypes
+import importlib
 import os
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libkvq.so")
 
 # The native host path: each function returns None for a call it does not take, which then
-# goes through the Python path. Without the built module every call does, and `lib` raises.
-try:
-    import torch  # noqa: F401  (the module links against torch's libraries)
-    from kvq_decode_amd import _host as host
-    HOST_BUILT = True
-except ImportError:
-    HOST_BUILT = False
+# goes through the Python path. Until `lib` has loaded both libraries it takes none.
+HOST_PATH = os.path.join(_PKG_DIR, "_host.so")
 
-    class host:  # noqa: N801
-        @staticmethod
-        def decode(*args):
-            return None
 
-        quantize = quantize_append = append_kv = reshape_and_cache = set_cu_count = decode
+class _NoHost:
+    @staticmethod
+    def decode(*args):
+        return None
+
+    quantize = quantize_append = append_kv = reshape_and_cache = set_cu_count = decode
+
+
+host = _NoHost
+_cu_counts = {}  # compute units by device index, as the native path has been told
+
+
+def __getattr__(name):
+    if name == "HOST_BUILT":  # asked each time: a build may come after the import
+        return os.path.exists(HOST_PATH)
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+
 
 # kvq_status (include/kvq.h)
 KVQ_OK = 0
@@ -155,11 +164,8 @@ def lib():
         L.kvq_reshape_and_cache.argtypes = [args_p, _vp, _vp, _i64, _i64, _vp, _i32, _vp]
         L.kvq_paged_decode_static.restype = ctypes.c_int
         L.kvq_paged_decode_static.argtypes = [args_p, _i32, _i32, _vp]
-        if not HOST_BUILT:
-            raise ImportError("kvq_decode_amd/_host.so is not built; run "
-                              "`python -m kvq_decode_amd.build`")
-        bind_host(L)
         _lib = L
+        _load_host(L)
     return _lib
 
 
@@ -169,9 +175,36 @@ HOST_SYMBOLS = ("kvq_head_blocks", "kvq_plan_decode", "kvq_plan_units", "kvq_nor
                 "kvq_quantize_append", "kvq_append_kv", "kvq_reshape_and_cache")
 
 
-def bind_host(L):
+def _load_host(L):
+    """Imports the native host path and binds it to the loaded library. It is loaded with the
+    library and not with the package, so that a build run from a process that has imported the
+    package is followed by the modules it built. The Python path is complete without it: one
+    that is missing or fails to load costs host time only, and is reported as a warning."""
+    global host
+    try:
+        import torch  # noqa: F401  (the module links against torch's libraries)
+        importlib.invalidate_caches()
+        module = importlib.import_module("kvq_decode_amd._host")
+        bind_host(L, module)
+    except Exception as e:
+        why = "is not built" if not os.path.exists(HOST_PATH) else f"does not load ({e})"
+        warnings.warn(f"{HOST_PATH} {why}: calls take the slower Python host path; run "
+                      "`python -m kvq_decode_amd.build`", RuntimeWarning, stacklevel=3)
+        return
+    host = module
+    for device, count in _cu_counts.items():
+        host.set_cu_count(device, count)
+
+
+def bind_host(L, module=None):
     """Points the native host path at the loaded library's functions."""
-    host.bind(*(ctypes.cast(getattr(L, name), _vp).value for name in HOST_SYMBOLS))
+    (module or host).bind(*(ctypes.cast(getattr(L, name), _vp).value for name in HOST_SYMBOLS))
+
+
+def set_cu_count(device, count):
+    """Tells the native host path a device's compute units, now or once it is loaded."""
+    _cu_counts[device] = count
+    host.set_cu_count(device, count)
 
 
 def check(func, status):

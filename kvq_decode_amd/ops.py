@@ -53,7 +53,7 @@ def _require(cond, msg):
 def _sm_count(device_index: int) -> int:
     """Compute units of the device (reference triton_fp16.py:170-172; 256 on MI355X)."""
     n = torch.cuda.get_device_properties(device_index).multi_processor_count
-    _lib.host.set_cu_count(device_index, n)
+    _lib.set_cu_count(device_index, n)
     return n
 
 
