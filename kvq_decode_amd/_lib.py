@@ -198,7 +198,7 @@ def _load_host(L):
 
 def bind_host(L, module=None):
     """Points the native host path at the loaded library's functions."""
-    (module or host).bind(*(ctypes.cast(getattr(L, name), _vp).value for name in HOST_SYMBOLS))
+    (module or host).bind(check, *(ctypes.cast(getattr(L, name), _vp).value for name in HOST_SYMBOLS))
 
 
 def set_cu_count(device, count):

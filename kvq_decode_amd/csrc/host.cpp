@@ -8,10 +8,11 @@
 //
 // Each returns None, having launched nothing, for a call it does not take: one that fails a
 // check, an argument of another Python type than the usual one (a numpy integer, a tensor
-// subclass, a tensor without storage), a q that needs a copy, a library status below zero.
+// subclass, a tensor without storage), a q that needs a copy, a call the library refuses.
 // The Python entry point then takes the call through its own path, which reports every error
 // and converts what can be converted; so the calls accepted and the errors raised are those of
-// the Python path. Nothing is kept from one call for the next.
+// the Python path. A failed launch (KVQ_ERR_HIP) is raised here: a kernel may be running, and
+// the error is reported once. Nothing is kept from one call for the next.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -44,8 +45,16 @@ struct Library {
 };
 Library L{};
 bool bound = false;
+PyObject* check_status = nullptr;  // _lib.check(func, status), which raises KvqError
 constexpr int kMaxDevices = 64;
 int32_t cu_count[kMaxDevices];
+
+// nullptr for a library status below zero: not taken, except a failed launch, whose KvqError
+// is set.
+PyObject* refused(const char* func, int status) {
+    if (status == KVQ_ERR_HIP) Py_XDECREF(PyObject_CallFunction(check_status, "si", func, status));
+    return nullptr;
+}
 
 // An ordinary GPU tensor: exactly torch.Tensor (or Parameter), strided, with storage of its
 // own; nullptr otherwise.
@@ -254,7 +263,7 @@ PyObject* decode(PyObject* const* o, Py_ssize_t n) {
     Py_BEGIN_ALLOW_THREADS;
     st = u > 0 ? L.decode_units(&a, u, opp, lsp, stream) : L.paged_decode(&a, s, opp, lsp, stream);
     Py_END_ALLOW_THREADS;
-    if (st < 0) return nullptr;
+    if (st < 0) return refused(u > 0 ? "kvq_decode_units" : "kvq_paged_decode", st);
     if (own_out.defined()) return THPVariable_Wrap(std::move(own_out));
     return Py_NewRef(o[13]);
 }
@@ -320,7 +329,7 @@ PyObject* quantize(PyObject* const* o, Py_ssize_t n) {
     st = L.quantize_cache(&a, k->data_ptr(), v->data_ptr(), k->stride(0), k->stride(1),
                           k->stride(2), stream);
     Py_END_ALLOW_THREADS;
-    return st < 0 ? nullptr : Py_NewRef(Py_True);
+    return st < 0 ? refused("kvq_quantize_cache", st) : Py_NewRef(Py_True);
 }
 
 // quantize_append(cache, k_new, v_new, block_table, seq_lens, k_resid)
@@ -342,7 +351,7 @@ PyObject* quantize_append(PyObject* const* o, Py_ssize_t n) {
     Py_BEGIN_ALLOW_THREADS;
     st = L.quantize_append(&a, kn->data_ptr(), vn->data_ptr(), res->data_ptr(), stream);
     Py_END_ALLOW_THREADS;
-    return st < 0 ? nullptr : Py_NewRef(Py_True);
+    return st < 0 ? refused("kvq_quantize_append", st) : Py_NewRef(Py_True);
 }
 
 // The fp16 caches of the append entry points (cache._cache_args).
@@ -375,7 +384,7 @@ PyObject* append_kv(PyObject* const* o, Py_ssize_t n) {
     Py_BEGIN_ALLOW_THREADS;
     st = L.append_kv(&a, kn->data_ptr(), vn->data_ptr(), stream);
     Py_END_ALLOW_THREADS;
-    return st < 0 ? nullptr : Py_NewRef(Py_True);
+    return st < 0 ? refused("kvq_append_kv", st) : Py_NewRef(Py_True);
 }
 
 // reshape_and_cache(key, value, k_cache, v_cache, slot_mapping)
@@ -403,7 +412,7 @@ PyObject* reshape_and_cache(PyObject* const* o, Py_ssize_t n) {
                              static_cast<const int64_t*>(slots->data_ptr()), int32_t(shape[0]),
                              stream);
     Py_END_ALLOW_THREADS;
-    return st < 0 ? nullptr : Py_NewRef(Py_True);
+    return st < 0 ? refused("kvq_reshape_and_cache", st) : Py_NewRef(Py_True);
 }
 
 // The Python-callable form: None for a call not taken. A C++ exception of torch (an
@@ -423,22 +432,25 @@ PyObject* entry(PyObject*, PyObject* const* o, Py_ssize_t n) {
     return r ? r : Py_NewRef(Py_None);
 }
 
-// bind(address, ...): libkvq.so's entry points in the order of Library's members
+// bind(check, address, ...): _lib.check, and libkvq.so's entry points in the order of
+// Library's members
 PyObject* bind(PyObject*, PyObject* const* o, Py_ssize_t n) {
     constexpr int kCount = sizeof(Library) / sizeof(void*);
-    if (n != kCount) {
-        PyErr_SetString(PyExc_TypeError, "bind takes one address per library entry point");
+    if (n != 1 + kCount || !PyCallable_Check(o[0])) {
+        PyErr_SetString(PyExc_TypeError,
+                        "bind takes the status check and one address per library entry point");
         return nullptr;
     }
     void* p[kCount];
     for (int i = 0; i < kCount; ++i) {
-        p[i] = PyLong_AsVoidPtr(o[i]);
+        p[i] = PyLong_AsVoidPtr(o[1 + i]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null entry point");
             return nullptr;
         }
     }
     memcpy(&L, p, sizeof(L));
+    Py_XSETREF(check_status, Py_NewRef(o[0]));
     bound = true;
     Py_RETURN_NONE;
 }

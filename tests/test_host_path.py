@@ -2,6 +2,7 @@
 
 The two must take the same calls with the same results and leave the same errors: the
 native functions return None for what they do not take, and the Python path then answers."""
+import ctypes
 import math
 
 import numpy as np
@@ -119,6 +120,7 @@ def test_decode_same_as_python_path(monkeypatch, lens, fmt):
 @pytest.mark.gpu
 def test_errors_same_as_python_path(monkeypatch):
     """Every refused call raises what it raises without the native path."""
+    _lib.lib()  # binds the library's functions
     q, k, v, bt, sl = _caches([300, 40], 16, 8, 2, 64)
     ws = (torch.empty(8, device="cuda"), torch.empty(8, device="cuda"))
     bad = [dict(q=q.float()), dict(k_cache=k.float()), dict(v_cache=v[1:]), dict(k_cache=k[..., :32]),
@@ -174,3 +176,53 @@ def test_write_paths_same_as_python_path(monkeypatch, fmt):
                     (reshape_and_cache, (rows[:, 1:4], rows[:, 5:8], k, v, slots))):
         with pytest.raises(KvqArgumentError):
             f(*args)
+
+
+@pytest.mark.gpu
+def test_launch_error_is_raised_after_one_call():
+    """A library function that reports a failed launch is called once and its status raised: a
+    second call through the Python path could return normally and hide it. The functions that
+    launch are host-side stand-ins here; no kernel runs."""
+    from kvq_decode_amd.cache import append_kv, reshape_and_cache
+    from kvq_decode_amd.quant import (allocate_quantized_cache, init_k_residual, quantize_append,
+                                      quantize_paged_cache)
+    q, k, v, bt, sl = _caches([300, 40], 16, 8, 2, 64)
+    new, slots = k[0, :2].contiguous(), torch.zeros(2, dtype=torch.int64, device="cuda")
+    qc = allocate_quantized_cache(k.shape[0], 16, 2, 64, "int8", "cuda")
+    resid = init_k_residual(k, bt, sl)
+    paged_decode_attention(q, k, v, bt, sl)  # the CU count of the device is known now
+    launches = ("kvq_paged_decode", "kvq_decode_units", "kvq_quantize_cache",
+                "kvq_quantize_append", "kvq_append_kv", "kvq_reshape_and_cache")
+    calls = []
+
+    class Failing:
+        """The library, with every launching function replaced."""
+        kept = []
+
+        def __getattr__(self, name):
+            f = getattr(_lib.lib(), name)
+            if name not in launches:
+                return f
+            params = [ctypes.c_void_p if t not in (ctypes.c_int32, ctypes.c_int64) else t
+                      for t in f.argtypes]
+            stub = ctypes.CFUNCTYPE(ctypes.c_int, *params)(
+                lambda *a: calls.append(name) or _lib.KVQ_ERR_HIP)
+            self.kept.append(stub)
+            return stub
+
+    try:
+        _lib.bind_host(Failing())
+        for name, call in (
+                ("kvq_paged_decode", lambda: paged_decode_attention(q, k, v, bt, sl, None, 1)),
+                ("kvq_decode_units", lambda: paged_decode_attention(q, k, v, bt, sl, units=3)),
+                ("kvq_quantize_cache", lambda: quantize_paged_cache(k, v, bt, sl, "int8", out=qc)),
+                ("kvq_quantize_append", lambda: quantize_append(qc, new, new, bt, sl, resid)),
+                ("kvq_append_kv", lambda: append_kv(k, v, new, new, bt, sl)),
+                ("kvq_reshape_and_cache", lambda: reshape_and_cache(new, new, k, v, slots))):
+            calls.clear()
+            with pytest.raises(_lib.KvqError) as e:
+                call()
+            assert calls == [name] and e.value.status == _lib.KVQ_ERR_HIP
+    finally:
+        _lib.bind_host(_lib.lib())
+    assert torch.equal(paged_decode_attention(q, k, v, bt, sl), paged_decode_attention(q, k, v, bt, sl))
