@@ -289,7 +289,9 @@ __device__ __forceinline__ void quant_k_group(const QuantParams& p, int kvh, int
     asm volatile("" : "+v"(lane));
     const int c = lane % PC, ri = lane / PC;
     const int n = seq_len_of(p, b);
-    const int t0 = grp * p.k_group, t1 = min(t0 + p.k_group, n);
+    // the launch's spare waves first: their groups may start past 2^31
+    if (grp >= p.max_groups) return;
+    const int t0 = grp * p.k_group, t1 = (int)min((uint32_t)t0 + (uint32_t)p.k_group, (uint32_t)n);
     if (t0 >= t1) return;  // uniform over the wave
     const int last = t1 - t0 - 1;  // the group's last row
     const int bmask = p.block_size - 1;
@@ -419,8 +421,8 @@ __device__ __forceinline__ void quant_v_tile(const QuantParams& p, int kvh, int 
     constexpr int LPR = D / 8, RPI = 64 / LPR, NI = kVIter<D>, ROWS = NI * RPI;
     const int lane = threadIdx.x & 63, c = lane % LPR, ri = lane / LPR;
     const int n = seq_len_of(p, b);
-    const int r0 = tile * ROWS;  // the wave's first row
-    if (r0 >= n) return;         // uniform over the wave
+    if ((int64_t)tile * ROWS >= n) return;  // uniform over the wave
+    const int r0 = tile * ROWS;             // the wave's first row
     const int last = min(ROWS, n - r0) - 1, last_blk = last / RPI;
     const int bmask = p.block_size - 1, vg = 1 << p.vg_shift;
     // lane j: page pg0 + j, pg0 the first page of the first row's V group

@@ -758,3 +758,20 @@ def test_append_moved_slices(fmt, D):
             for name in ("k_scale", "k_zero"):
                 g, w = (getattr(c, name).cpu().numpy()[lead].view(np.uint16) for c in (got, want))
                 assert np.array_equal(g, w), f"{name} k_group={k_group} rows={rows} moved={nm}"
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_bulk_quantizer_huge_k_group(fmt):
+    """A K group far longer than the table: one group per sequence, as a group of the table's
+    length gives, also where the launch's spare waves hold groups that would start past 2^31
+    (2^30: the third; 2^31 - 64: the second)."""
+    from kvq_decode_amd.quant import allocate_quantized_cache, quantize_paged_cache
+    q, kc, vc, bt, sl = make([300, 70], 16, Hq=2, Hkv=2, D=128, seed=9)
+    got = []
+    for k_group in (512, 2**30, 2**31 - 64):
+        out = allocate_quantized_cache(kc.shape[0], 16, 2, 128, fmt, "cuda", k_group)
+        for t in out[:6]:
+            t.zero_()
+        quantize_paged_cache(gpu(kc), gpu(vc), gpu(bt), gpu(sl), fmt, k_group=k_group, out=out)
+        got.append([t.cpu().numpy().tobytes() for t in out[:6]])
+    assert got[0] == got[1] == got[2]
