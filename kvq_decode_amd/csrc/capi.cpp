@@ -242,7 +242,8 @@ int check_quant_args(const kvq_decode_args* a) {
     if (a->head_dim != 64 && a->head_dim != 128 && a->head_dim != 256) return KVQ_ERR_UNSUPPORTED;
     if (a->k_group < a->block_size || a->k_group % a->block_size != 0) return KVQ_ERR_UNSUPPORTED;
     if (a->batch > 65535 || a->kv_heads > 65535) return KVQ_ERR_UNSUPPORTED;
-    // 1-D grids over (kv head, K group) and (kv head, 64-row tile); tokens are int32
+    // tokens are int32; a bound on the bulk launch's 1-D grid (K groups and V tiles of every kv
+    // head), whose exact size the launch checks
     const int64_t tokens = int64_t(a->max_blocks) * a->block_size;
     if (tokens > INT32_MAX || int64_t(a->kv_heads) * ((tokens + 63) / 64) > INT32_MAX)
         return KVQ_ERR_UNSUPPORTED;

@@ -264,6 +264,13 @@ __device__ __forceinline__ void store_pairs8(_Float16* dst, const ScaleZero* q) 
     *(u4q*)(dst + 8) = u4q{q[4].sz, q[5].sz, q[6].sz, q[7].sz};
 }
 
+// K groups of one wave (at head dim 256: of two, 128 channels each): the whole groups within
+// kSmallSpan tokens, or one larger group.
+constexpr int kSmallSpan = 64;
+__host__ __device__ inline int k_groups_per_wave(int k_group) {
+    return k_group <= kSmallSpan ? kSmallSpan / k_group : 1;
+}
+
 // K, bulk: one wave per (group, 128 channels of a kv head, sequence): the group's rows in
 // slabs of 128, 8 chunks of 16 rows (a chunk lies in one page). A load instruction covers RPI
 // whole rows (PC lanes of 16 bytes each): lane (ri, c) owns channels 8c .. 8c + 7 of rows
@@ -274,7 +281,8 @@ __device__ __forceinline__ void store_pairs8(_Float16* dst, const ScaleZero* q) 
 // base per chunk plus the lane's offset. Where a slab is cut short or a page lies outside the
 // pool, the missing rows are replaced by rows of the group that count, which leave its min /
 // max as they are, and are not written. Min / max run on packed halves, over the rows in
-// registers and then across the RPI lanes that share channels: no LDS, no barrier. Codes go
+// registers and then across the RPI lanes that share channels: no LDS, no barrier. Row limits
+// are compared with ri itself: RPI i + ri, kept in registers over the loops, would spill. Codes go
 // to each token's page slot, the pairs to the group's first page; a group whose first page
 // lies outside the pool could not be read back and writes nothing.
 template <int FMT, int D>
@@ -282,12 +290,7 @@ __device__ __forceinline__ void quant_k_group(const QuantParams& p, int kvh, int
                                               int b) {
     constexpr int CW = D < 128 ? D : 128;  // channels of a wave
     constexpr int PC = CW / 8, RPI = 64 / PC, KC = 128 / RPI, CI = 16 / RPI;
-    int lane = threadIdx.x & 63;
-    // opaque, so that the lane's addresses are not kept in registers across the caller's loop
-    // over groups (the rows already fill the file: spills, 82.5 -> 86.9 us with the INT4 case
-    // of quant_bulk_kernel)
-    asm volatile("" : "+v"(lane));
-    const int c = lane % PC, ri = lane / PC;
+    const int lane = threadIdx.x & 63, c = lane % PC, ri = lane / PC;
     const int n = seq_len_of(p, b);
     // the launch's spare waves first: their groups may start past 2^31
     if (grp >= p.max_groups) return;
@@ -333,7 +336,7 @@ __device__ __forceinline__ void quant_k_group(const QuantParams& p, int kvh, int
                     if (kk != k) continue;  // static register indices
 #pragma unroll
                     for (int i = 0; i < CI; ++i)
-                        rows[CI * kk + i] = load_nt(base + (int64_t)min(RPI * i + ri, last - r0) * p.s_stok);
+                        rows[CI * kk + i] = load_nt(base + (int64_t)(RPI * i + min(ri, last - r0 - RPI * i)) * p.s_stok);
                 }
             }
         }
@@ -376,12 +379,93 @@ __device__ __forceinline__ void quant_k_group(const QuantParams& p, int kvh, int
 #pragma unroll
             for (int i = 0; i < CI; ++i) {
                 const Codes8<FMT> w = encode8<FMT, 1>(rows[CI * k + i], q, live);
-                if (RPI * i + ri <= last - r0) store8<FMT, true>(base + RPI * i * p.k_stok, w);
+                if (ri <= last - r0 - RPI * i) store8<FMT, true>(base + RPI * i * p.k_stok, w);
             }
         }
         if (--s < 0) break;
         pages = slab_pages(128 * s);
         fill(128 * s);
+    }
+}
+
+// K, bulk, groups of up to kSmallSpan tokens: one wave per (whole groups of that many tokens
+// together, 128 channels of a kv head, sequence). The rows are loaded all at once, as
+// quant_k_group's slab, and then group by group reduced and encoded from their registers. A chunk
+// past the sequence or in a page outside the pool is skipped in every pass (uniform over the
+// wave); the rows past the sequence in its last chunk are replaced by its last row and not
+// written.
+// Bound by HBM on large inputs, as the other groups (16 x 8192 tokens, 8 kv heads, D = 128, INT8,
+// groups of 16: 172 us, of 128: 165), and else by the chain of loads, reductions and stores, which
+// grows with the groups of a wave: 64 tokens and not 128, which halve the waves of a short batch
+// and at D >= 128 spill 26 registers (64: four waves per SIMD without spills). 64 sequences of 10 to 577 tokens, D = 256, INT8,
+// groups of 16: 65 us; one wave per group loading its 16 rows 74, eight groups one after the other
+// on a wave, each with a slab's loads, 304.
+template <int FMT, int D>
+__device__ __forceinline__ void quant_k_small(const QuantParams& p, int kvh, int span, int half,
+                                              int b) {
+    constexpr int CW = D < 128 ? D : 128;  // channels of a wave
+    constexpr int PC = CW / 8, RPI = 64 / PC, CI = 16 / RPI, NC = kSmallSpan / 16, KC = NC * CI;
+    const int lane = threadIdx.x & 63, c = lane % PC, ri = lane / PC;
+    const int n = seq_len_of(p, b);
+    const int per = k_groups_per_wave(p.k_group), len = per * p.k_group, gc = p.k_group / 16;
+    if ((int64_t)span * len >= n) return;  // uniform over the wave
+    const int t0 = span * len, last = min(len, n - t0) - 1;  // the span's last row
+    const int bmask = p.block_size - 1;
+    // lane j: the page of chunk j % NC (-1: outside the pool, or no chunk of the span)
+    int pages = phys_of(p, b, (t0 + min(16 * (lane % NC), last)) >> p.bs_shift);
+    if (16 * (lane % NC) > last) pages = -1;
+    const int ch = half * CW + 8 * c;  // the lane's first channel
+    const _Float16* src = p.k_src + (int64_t)kvh * p.s_sh + ch;
+    h8q rows[KC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const int ph = __builtin_amdgcn_readlane(pages, k);
+        if (ph < 0) continue;
+        const _Float16* base = src + (int64_t)ph * p.s_sblk + (int64_t)((t0 + 16 * k) & bmask) * p.s_stok;
+#pragma unroll
+        for (int i = 0; i < CI; ++i)
+            rows[CI * k + i] = load_nt(base + (int64_t)min(RPI * i + ri, last - 16 * k) * p.s_stok);
+    }
+    constexpr int CB = FMT == KVQ_KV_INT4 ? 4 : 8;  // code bytes per lane and row
+    uint8_t* dst = p.k_codes + (int64_t)kvh * p.k_sh + ch / 8 * CB + (int64_t)ri * p.k_stok;
+    for (int c0 = 0; 16 * c0 <= last; c0 += gc) {  // the group of chunks c0 .. c0 + gc - 1
+        const int lead = __builtin_amdgcn_readlane(pages, c0);
+        if (lead < 0) continue;
+        h8q mn, mx;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            mn[e] = (_Float16)INFINITY;
+            mx[e] = (_Float16)-INFINITY;
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            if (k < c0 || k >= c0 + gc || __builtin_amdgcn_readlane(pages, k) < 0) continue;
+#pragma unroll
+            for (int i = 0; i < CI; ++i) {
+                mn = __builtin_elementwise_min(mn, rows[CI * k + i]);
+                mx = __builtin_elementwise_max(mx, rows[CI * k + i]);
+            }
+        }
+        if constexpr (PC <= 8) minmax8_xor<8>(mn, mx);
+        minmax8_xor<16>(mn, mx);
+        minmax8_xor<32>(mn, mx);
+        ScaleZero q[8];
+        uint32_t live[2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = make_params<FMT>((float)mn[e], (float)mx[e]);
+        live_masks<FMT>(q, live);
+        if (ri == 0) store_pairs8(p.k_scale + 2 * (((int64_t)lead * p.kv_heads + kvh) * D + ch), q);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const int ph = __builtin_amdgcn_readlane(pages, k);
+            if (k < c0 || k >= c0 + gc || ph < 0) continue;
+            uint8_t* base = dst + (int64_t)ph * p.k_sblk + (int64_t)((t0 + 16 * k) & bmask) * p.k_stok;
+#pragma unroll
+            for (int i = 0; i < CI; ++i) {
+                const Codes8<FMT> w = encode8<FMT, 1>(rows[CI * k + i], q, live);
+                if (RPI * i + ri <= last - 16 * k) store8<FMT, true>(base + RPI * i * p.k_stok, w);
+            }
+        }
     }
 }
 
@@ -620,13 +704,6 @@ __device__ __forceinline__ void quant_k_append(const QuantParams& p, int kvh, in
     }
 }
 
-// Waves of a (kv head, sequence) per 4-wave K workgroup's share: a wave takes one K group, or
-// the groups of 128 tokens when they are smaller; at head dim 256 two waves share a group
-// (128 channels each).
-__host__ __device__ inline int k_groups_per_wave(int k_group) {
-    return k_group < 128 ? 128 / k_group : 1;
-}
-
 // Bulk, one launch: the K groups and the V row tiles of every (kv head, sequence), in 4-wave
 // workgroups; per (kv head, sequence) kb K and vb V workgroups, alternating through the grid
 // (of every kb + vb consecutive, kb are K), so that both kinds are in flight together and the
@@ -643,7 +720,8 @@ __host__ __device__ inline int k_groups_per_wave(int k_group) {
 // instead of 8 83.9 / 172.5 (32: 90.7); the XCD order 83.4 / 166.1; fewer registers (s and z
 // in one) 82.5 / 164.5. 4 waves per SIMD spill (126.9 / 256.1). All V workgroups after the K
 // ones: 86.2 / 165.8.
-template <int FMT, int D>
+// SMALL: K groups of up to kSmallSpan tokens.
+template <int FMT, int D, bool SMALL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 void quant_bulk_kernel(const QuantParams p, int kb, int vb) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -659,10 +737,10 @@ void quant_bulk_kernel(const QuantParams p, int kb, int vb) {
     }
     const int k0 = (int)((int64_t)j * kb / nb), k1 = (int)((int64_t)(j + 1) * kb / nb);
     if (k1 > k0) {
-        constexpr int PER = D > 128 ? D / 128 : 1;  // waves per group
-        const int w = 4 * k0 + wave, per = k_groups_per_wave(p.k_group);
-        for (int g = 0; g < per; ++g)
-            quant_k_group<FMT, D>(p, kvh, w / PER * per + g, w % PER, b);
+        constexpr int PER = D > 128 ? D / 128 : 1;  // waves per group or span
+        const int w = 4 * k0 + wave;
+        if constexpr (SMALL) quant_k_small<FMT, D>(p, kvh, w / PER, w % PER, b);
+        else quant_k_group<FMT, D>(p, kvh, w / PER, w % PER, b);
     } else {
         quant_v_tile<FMT, D>(p, kvh, 4 * (j - k0) + wave, b);
     }
@@ -692,8 +770,9 @@ hipError_t launch_fmt_d(const QuantParams& p, hipStream_t stream) {
     const int per = k_groups_per_wave(p.k_group);
     const int kb = (PER * ((p.max_groups + per - 1) / per) + 3) / 4;
     const int vb = (int)(((int64_t)p.max_blocks * p.block_size + VROWS - 1) / VROWS);
-    hipLaunchKernelGGL((quant_bulk_kernel<FMT, D>), dim3(p.kv_heads * (kb + vb), p.batch),
-                       dim3(256), 0, stream, p, kb, vb);
+    if (int64_t(p.kv_heads) * (int64_t(kb) + vb) > INT32_MAX) return hipErrorInvalidConfiguration;
+    const auto kernel = p.k_group <= kSmallSpan ? quant_bulk_kernel<FMT, D, true> : quant_bulk_kernel<FMT, D, false>;
+    hipLaunchKernelGGL(kernel, dim3(p.kv_heads * (kb + vb), p.batch), dim3(256), 0, stream, p, kb, vb);
     return hipGetLastError();
 }
 

@@ -775,3 +775,40 @@ def test_bulk_quantizer_huge_k_group(fmt):
         quantize_paged_cache(gpu(kc), gpu(vc), gpu(bt), gpu(sl), fmt, k_group=k_group, out=out)
         got.append([t.cpu().numpy().tobytes() for t in out[:6]])
     assert got[0] == got[1] == got[2]
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_bulk_quantizer_small_k_groups(fmt, D):
+    """K groups of up to 64 tokens, several to a wave, and the sizes just above: every byte of
+    the K codes and pairs, at lengths one short of, equal to and one past a chunk, a group and a
+    wave's span (48 or 64 tokens), with block-table entries outside the pool. Their rows enter no
+    range and are not written, and a group that starts in one is not written at all."""
+    from kvq_decode_amd.quant import allocate_quantized_cache, quantize_paged_cache
+    lens, hkv = [1, 15, 16, 17, 47, 48, 49, 63, 64, 65, 97, 128, 145, 200], 3
+    for bs, k_group in ((16, 16), (16, 32), (16, 48), (32, 32), (16, 64), (64, 64), (16, 80), (16, 112)):
+        q, kc, vc, bt, sl = make(lens, bs, Hq=hkv, Hkv=hkv, D=D, seed=bs + k_group + D)
+        nb = kc.shape[0]
+        if bs == 16:  # the first, an inner and the last page of a group, of a span, of a table row
+            for b, page in ((4, 1), (5, 2), (9, 4), (10, 0), (11, 3), (11, 7), (12, 4), (13, 5), (13, 8)):
+                bt[b, page] = -1 if b % 2 else nb
+        got = allocate_quantized_cache(nb, bs, hkv, D, fmt, "cuda", k_group)
+        for t in got[:6]:
+            t.fill_(7)
+        quantize_paged_cache(gpu(kc), gpu(vc), gpu(bt), gpu(sl), fmt, k_group=k_group, out=got)
+        want = {n: getattr(got, n).cpu().numpy() * 0 + 7 for n in ("k_codes", "k_scale", "k_zero")}
+        for b, n in enumerate(lens):
+            for t0 in range(0, n, k_group):
+                lead = bt[b, t0 // bs]
+                if not 0 <= lead < nb:
+                    continue
+                at = [(bt[b, t // bs], t % bs) for t in range(t0, min(t0 + k_group, n))]
+                page, slot = np.array([a for a in at if 0 <= a[0] < nb]).T
+                x = kc[page, slot]
+                s, z = kivi.params(x.min(axis=0), x.max(axis=0), fmt)
+                want["k_scale"][lead], want["k_zero"][lead] = s, z
+                c = kivi.codes(x, s[None], z[None], fmt)
+                want["k_codes"][page, slot] = kivi.pack_int4(c) if fmt == "int4" else c
+        for name, w in want.items():
+            g = getattr(got, name).cpu().numpy()
+            assert g.tobytes() == w.tobytes(), f"{name} D={D} bs={bs} k_group={k_group}"
