@@ -155,7 +155,8 @@ def build_checks(verbose=False):
         src = os.path.join(CHECKS_DIR, name)
         out = src[:-len(".hip")]
         cmd = [hipcc(), f"--offload-arch={ARCH}", "-O3", "-std=c++17",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", src, "-o", out]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+               f"-I{INCLUDE}", f"-I{CSRC}", src, "-o", out]
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError("hipcc failed (%d) on %s:\n%s"

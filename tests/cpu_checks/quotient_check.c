@@ -1,4 +1,4 @@
-/* CPU check of the quantizers' quotient (kvq_decode_amd/csrc/quant.hip, quotient()):
+/* CPU check of the quantizers' quotient (kvq_decode_amd/csrc/quant_math.h, quotient()):
  *   r = RN(1/s), q = RN(d r), rem = fma(-q, s, d), t = fma(rem, r, q)
  * must equal the IEEE quotient RN(d / s) bit for bit for every positive finite fp16 s and
  * every d = fl32(x - z) of fp16 x, z (0 or |d| >= 2^-24). Cases: random fp16 x, z for

@@ -1,5 +1,5 @@
-// Exhaustive check of the quantizers' e4m3fn encode (kvq_decode_amd/csrc/quant.hip
-// e4m3fn_rne: the hardware conversion v_cvt_scalef32_pk_fp8_f32 at scale 1) against the
+// Exhaustive check of the quantizers' e4m3fn encode (kvq_decode_amd/csrc/quant_math.h
+// encode8: the hardware conversion v_cvt_scalef32_pk_fp8_f32 at scale 1) against the
 // spec's software encode (oracle/kivi.py: mantissa rounded half to even at 2^(e-3),
 // subnormals at 2^-9), for every fp32 bit pattern in [0, 448] and its negation
 // (2,277,507,074 values). Prints the count of differences and the first few; exit status 0
@@ -41,7 +41,7 @@ __device__ uint32_t spec_e4m3fn(float t) {
     return bits | sign;
 }
 
-// The kernel's encode (quant.hip).
+// The kernel's conversion (quant_math.h).
 __device__ uint32_t kernel_e4m3fn(float t) {
     const s2 r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(s2{0, 0}, t, 0.f, 1.0f, false);
     return __builtin_bit_cast(uint32_t, r) & 0xFFu;

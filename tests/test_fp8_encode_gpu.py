@@ -1,4 +1,4 @@
-"""The quantizers' FP8 encode (the hardware e4m3fn conversion in quant.hip) equals the
+"""The quantizers' FP8 encode (the hardware e4m3fn conversion in quant_math.h) equals the
 spec's software encode on every fp32 value of [-448, 448]: tests/gpu_checks/
 fp8_encode_check.hip compares the two over all 2,277,507,074 of them on the GPU. The
 quantizer itself is held to the numpy spec by tests/test_quant_gpu.py, including the e4m3

@@ -1,12 +1,13 @@
-"""The quantizers' division shortcut is the IEEE quotient on their whole input domain.
+"""The quantizers' division shortcut is the IEEE quotient, on random and near-tie inputs.
 
-quant.hip computes the spec's correctly rounded t = RN((x - z) / s) as RN(d r) plus one
+quant_math.h computes the spec's correctly rounded t = RN((x - z) / s) as RN(d r) plus one
 fma remainder and one fma correction, with r = RN(1 / s) (Markstein's theorem; its
 exceptions need a 24-ones divisor significand, and s is an fp16 value). The C program
 tests/cpu_checks/quotient_check.c compares that sequence with IEEE division bit for bit
 for every finite fp16 s (about 4 million cases); the planted variant without the
-correction must fail, which shows the check can see a difference. The GPU kernels
-themselves are held to the numpy spec bit for bit by tests/test_quant_gpu.py.
+correction must fail, which shows the check can see a difference. The codes it gives on the
+GPU are checked by tests/test_quant_math_gpu.py, the kernels against the numpy spec by
+tests/test_quant_gpu.py.
 """
 import os
 import shutil
