@@ -198,9 +198,9 @@ int kvq_plan_decode(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t bl
  *           T = 4 s, waves = 4; INT4 T = 8 s, waves = min(2 s, 4)
  *           (s as in kvq_plan_decode),
  * for kvq_decode_units; otherwise units = waves = 0 (use kvq_plan_decode's split plan).
- * Short partitions take the split plan too, whose workgroups start faster: at most 16 chunks
- * (head_dim 256: 8) of a full table row per wave of it, at least 2 waves per CU in all and,
- * for fp16 head dims below 128, a workgroup per CU.
+ * Short partitions take the split plan too, whose workgroups start faster: batch >= 8, at most
+ * 16 chunks (head_dim 64 and 128; else 8) of a full table row per wave of it, at least 2 waves
+ * per CU in all and, for fp16 head dims below 128, a workgroup per CU.
  * As in kvq_plan_decode, waves is halved (and units doubled) until a workgroup's LDS fits
  * 64 KB, and q_heads / kv_heads must be 1..16.
  * Units balance ragged batches (a static split count sizes every sequence's splits by

@@ -379,18 +379,23 @@ int64_t head_dim_scale(int32_t head_dim) {
     return head_dim >= 128 ? 1 : head_dim >= 64 ? 128 / head_dim : 64 / head_dim;
 }
 
-// Short partitions: batches whose split plan leaves a wave at most 16 16-token chunks of a
-// full block-table row (head_dim 256, twice the bytes, and 16 and 32, whose units start faster:
-// 8) take splits instead of work units, from 8 sequences on (smaller batches keep units: the
-// captured model steps of 4 sequences are tested to run them). A
-// unit's start (the lengths scanned, its sequence searched, q and pages loaded for each of its
-// segments) then outweighs the balance it gives. Not below two waves per CU, where the cap on
-// splits leaves the CUs idle and units, as short as one chunk, are up to 1.5 times as fast.
+// Short partitions: batches of 8 and more sequences whose split plan leaves a wave at most 16
+// 16-token chunks of a full block-table row (head_dim 256, twice the bytes, and 16 and 32, whose
+// units start faster: 8) take splits instead of work units. A unit's start (the lengths scanned,
+// its sequence searched, q and pages loaded for each of its segments) then outweighs the balance
+// it gives. Not below two waves per CU, where the cap on splits leaves the CUs idle and units, as
+// short as one chunk, are up to 1.5 times as fast.
 // Measured on MI355X, us per call of units and splits (contexts from 1/8 of the longest):
 // 16 chunks per wave fp16 B8 x 2k 16.1 / 14.4, INT8 B16 x 2k 24.0 / 17.4, INT4 B8 x 8k
 // 22.8 / 17.2; 32: fp16 B8 x 4k 21.2 / 22.3, INT8 B8 x 8k 24.9 / 25.4. In a table two
 // to three times as wide as the longest context: 12 to 13 chunks per wave INT8 B8 x 1k 16.9 /
-// 14.9, FP8 B8 x 1.7k 16.2 / 16.7; 24: fp16 B8 x 1k 15.8 / 17.8.
+// 14.9, FP8 B8 x 1.7k 16.2 / 16.7; 24: fp16 B8 x 1k 15.8 / 17.8. Over 350 drawn shapes that the
+// rule moves (8 to 300 sequences, uniform to 1 long among short, tables up to ten times as wide as
+// the contexts) splits take 0.59 of the units' time on average and at most 1.10 (FP8, head_dim 256,
+// 16 q heads, a table ten times as wide: 20.9 / 23.1). Below 8 sequences they gain less, 0.79 over
+// 200 shapes, and lose more, in wide tables: 12 of the 200 by 1.05 to 1.22 (INT8, head_dim 256,
+// B2 x 71 tokens: 9.6 / 11.7). Those keep units, which the captured model steps of 4 sequences
+// are also tested to run.
 bool short_partitions(int64_t batch, int64_t pairs, int64_t chunks, int64_t per_pair,
                       int32_t head_dim, int32_t cu_count) {
     return batch >= 8 && pairs * per_pair >= 2 * int64_t(cu_count) &&

@@ -88,9 +88,10 @@ def plan_decode(batch: int, kv_heads: int, block_size: int, max_pages: int,
     512 (fp16) / 256 or, for batches whose (sequence, kv head) pairs outnumber the CUs, 64
     (quantized) 16-token chunks per wave; up to 2 waves per workgroup for fp16, and for
     quantized caches one wave per 8 waves of the (sequence, kv head) pair, up to 4 (INT4:
-    8; short partitions, see `plan_units`, at least 4). fp16 head dims below 128 get 128 / head_dim times the waves (16 and 32, whose rows
-    share lines between kv heads: 64 / head_dim), in workgroups of up to 4 waves. Waves are halved (splits doubled) until a workgroup's LDS, which grows with
-    the q heads per kv head, fits 64 KB. `kv_heads` counts the kernels' kv heads (see
+    8; short partitions, see `plan_units`, at least 4). fp16 head dims below 128 get 128 /
+    head_dim times the waves (16 and 32, whose rows share lines between kv heads: 64 /
+    head_dim), in workgroups of up to 4 waves. Waves are halved (splits doubled) until a
+    workgroup's LDS, which grows with the q heads per kv head, fits 64 KB. `kv_heads` counts the kernels' kv heads (see
     `head_blocks`); `q_heads` (default: kv_heads, one q head per kv head) all q heads."""
     _require(kv_format in KV_FORMATS, f"kv_format must be one of {tuple(KV_FORMATS)}")
     s, w = ctypes.c_int32(), ctypes.c_int32()
@@ -130,10 +131,11 @@ def plan_units(batch: int, kv_heads: int, block_size: int, max_pages: int,
     unit workgroups (fp16), 4 in 4-wave workgroups (INT8, FP8) or 8 in 2-wave workgroups
     (INT4), which keeps ragged batches balanced. Head dims below 128 get 128 / head_dim
     times the waves per CU (16 and 32: 64 / head_dim), and fp16 / INT4 unit workgroups of up
-    to 4 waves. Short partitions (at most 16 chunks per wave of the split plan, 8 at head
-    dim 256, in at least 2 waves per CU) take the split plan, whose workgroups start
-    faster. As in `plan_decode`, waves are halved (units doubled) until a workgroup's LDS fits 64 KB, and
-    `q_heads` defaults to kv_heads."""
+    to 4 waves. Short partitions (batches of 8 and more, at most 16 chunks per wave of the
+    split plan at head dims 64 and 128, else 8, in at least 2 waves per CU and, for fp16 head
+    dims below 128, at least a workgroup per CU) take the split plan, whose workgroups start
+    faster. As in `plan_decode`, waves are halved (units doubled) until a workgroup's LDS fits
+    64 KB, and `q_heads` defaults to kv_heads."""
     _require(kv_format in KV_FORMATS, f"kv_format must be one of {tuple(KV_FORMATS)}")
     u, w = ctypes.c_int32(), ctypes.c_int32()
     _lib.check("kvq_plan_units",
@@ -264,7 +266,7 @@ def paged_decode_attention(
     `units_workspace_shapes(B, Hq, D, units)`; with num_splits=None,
     `plan_workspace_shapes` gives whichever the plan needs). With num_splits=None the partition comes
     from `plan_units` (work units: batches of 2 to 1024 with 4096-token contexts or that the
-    split plan would split) or else `plan_decode` (`choose_num_splits` keeps the reference's formula for callers
+    split plan would split, except short partitions) or else `plan_decode` (`choose_num_splits` keeps the reference's formula for callers
     that want it). `units` > 0 (B <= 1024) asks for the work-unit partition: per kv head,
     all sequences' 16-token chunks in batch order cut into `units` equal ranges
     (`kvq_decode_units`)."""

@@ -242,9 +242,30 @@ def test_plan_short_partitions(fmt, hd, batch, edge):
     assert plan_units(batch, 8, 16, edge + 1, 256, fmt, hd, 32)[0] > 0
     splits, waves = plan_decode(batch, 8, 16, edge, 256, fmt, hd, 32)
     assert splits * waves * batch * 8 >= 512 and waves >= (2 if fmt == "fp16" else 4)
-    # 8 chunks per wave, but 256 waves on 256 CUs; fewer than 8 sequences: work units
-    assert plan_units(8, 8, 16, 16, 256, fmt, hd, 32)[0] > 0 or fmt == "fp16"
+    # fewer than 8 sequences: work units
     assert plan_units(4, 8, 16, edge, 256, fmt, hd, 32)[0] > 0
+
+
+@pytest.mark.parametrize("fmt,hd,units,first", [
+    ("fp16", 128, (256, 2), 256),
+    ("fp16", 256, (256, 2), 256),
+    ("fp16", 64, (256, 4), 512),   # at 256 pages 512 waves, but 128 workgroups
+    ("fp16", 32, (256, 4), 512),
+    ("int8", 128, (256, 4), 256),
+    ("fp8_e4m3", 64, (512, 4), 256),
+    ("int4", 128, (1024, 2), 256),
+])
+def test_plan_short_partitions_need_two_waves_per_cu(fmt, hd, units, first):
+    """8 sequences of one kv head, at most 8 chunks per wave: work units while the splits, capped
+    by the chunks, are fewer than 512 waves on 256 CUs (fp16 head dims below 128: or fewer than 256
+    workgroups), and splits from `first` pages on."""
+    from kvq_decode_amd.ops import plan_decode, plan_units
+    for pages in (64, 128, 255, 256, 512):
+        splits, waves = plan_decode(8, 1, 16, pages, 256, fmt, hd, 4)
+        assert pages <= 8 * splits * waves
+        enough = 8 * splits * waves >= 512 and (hd >= 128 or fmt != "fp16" or 8 * splits >= 256)
+        assert enough == (pages >= first)
+        assert plan_units(8, 1, 16, pages, 256, fmt, hd, 4) == ((0, 0) if enough else units)
 
 
 def test_plan_lds_budget():
