@@ -570,14 +570,15 @@ __device__ __forceinline__ void quant_k_append(const QuantParams& p, int kvh, in
 //
 // Bound by HBM, reads and writes mixed: without the arithmetic it takes 96 to 98% of the
 // time, and FP8 moves 4.9 TB/s where a plain copy moves 4.8. Measured (us per call, 8 kv
-// heads, D = 128): INT4, 8 sequences of 1000 to 16400 tokens, 126.4 -> 82.5; FP8, 16 x 8192,
-// 217.9 -> 164.5, against two kernels (K, then V) at about 20 VALU instructions per value. Of
+// heads, D = 128): INT4, 8 sequences of 1000 to 16400 tokens, 128.5 -> 78.3; FP8, 16 x 8192,
+// 218.4 -> 163.0, against two kernels (K, then V) at about 20 VALU instructions per value. Of
 // that, with the arithmetic above: one launch 98.6 / 186.6; 3 waves per SIMD (168 VGPRs, 172
 // without the attribute) 88.8 / 181.9; streaming stores 86.9 / 173.2; 16 V row blocks per wave
 // instead of 8 83.9 / 172.5 (32: 90.7); the XCD order 83.4 / 166.1; fewer registers (s and z
-// in one) 82.5 / 164.5. 4 waves per SIMD spill (126.9 / 256.1). All V workgroups after the K
-// ones: 86.2 / 165.8.
-// SMALL: K groups of up to kSmallSpan tokens.
+// in one) 82.5 / 164.5, (row limits, no loop over groups) 79.1 / 163.0. 4 waves per SIMD spill
+// (126.9 / 256.1). All V workgroups after the K ones: 86.2 / 165.8.
+//
+// SMALL: K groups of up to kSmallSpan tokens, a kernel of its own for its registers.
 template <int FMT, int D, bool SMALL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 void quant_bulk_kernel(const QuantParams p, int kb, int vb) {
